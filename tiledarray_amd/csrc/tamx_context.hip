@@ -4,6 +4,7 @@
 #include <new>
 
 #include "tamx_internal.hpp"
+#include "tamx_queue.hpp"
 
 namespace tamx {
 
@@ -122,13 +123,12 @@ int tamx_worklist_create(tamx_context* ctx, int64_t task_capacity,
   // search over item_prefix inside the GEMM kernel
   wl->item_capacity = std::min<int64_t>(tc * 16, (int64_t(1) << 31) - 1);
   alloc(&wl->item_task, sizeof(int32_t) * wl->item_capacity);
-  alloc(&wl->queue, sizeof(int32_t) * 16);
+  alloc(&wl->queue, sizeof(int32_t) * tamx::kQueueInts);
   // one partial per work-list workgroup (32 result tiles each), at least
   // one per item-planner chunk
   const int64_t nparts = std::max<int64_t>(tamx::kScanBlocks, gc / 32 + 1) + 1;
   alloc(reinterpret_cast<char**>(&wl->scan_partials), 32 * nparts);
   if (e == hipSuccess) e = hipMemset(wl->counters, 0, sizeof(int64_t) * TAMX_WL_NCOUNTERS);
-  if (e == hipSuccess) e = hipMemset(wl->queue, 0, sizeof(int32_t) * 16);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e != hipSuccess) {
     tamx::set_error(std::string("worklist allocation: ") + hipGetErrorString(e));

@@ -1,6 +1,7 @@
 // Plain entry points of the grouped GEMM and its item planner (the kernel
 // is in tamx_gemm.hpp).
 #include "tamx_gemm.hpp"
+#include "tamx_queue.hpp"
 #include "tamx_scan.hpp"
 
 namespace {
@@ -8,7 +9,8 @@ namespace {
 // Item planner: prefix[t] = number of BM x BN macro tiles of tasks 0..t-1,
 // and the item -> task map when it fits in item_capacity entries.  Three
 // launches (chunk sums over kScanBlocks workgroups, one-workgroup scan of the
-// sums, chunk rescans), each walking the task list once.
+// sums, chunk rescans), each walking the task list once.  The last one also
+// clears the item queue for the GEMM that follows.
 __device__ inline int64_t planned_tasks(const int64_t* counters, int64_t capacity) {
   const int64_t n = counters[TAMX_WL_NTASKS];
   return (n < 0 || n > capacity || counters[TAMX_WL_STATUS] != 0) ? 0 : n;
@@ -39,7 +41,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_items_fill_kernel(
     const tamx_gemm_task* __restrict__ tasks, const int64_t* __restrict__ counters,
     int bm, int bn, int64_t capacity, const int32_t* __restrict__ partial,
     int32_t* __restrict__ prefix, int32_t* __restrict__ item_task,
-    int64_t item_capacity) {
+    int64_t item_capacity, int32_t* __restrict__ queue) {
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < tamx::kQueueInts; i += kPlanThreads) queue[i] = 0;
   __shared__ int32_t part[kPlanThreads];
   const int64_t n = planned_tasks(counters, capacity);
   const int32_t total = partial[tamx::kScanBlocks];
@@ -69,7 +73,7 @@ int tamx::plan_items(tamx_worklist* wl, int bm, int bn, hipStream_t s) {
   TAMX_LAUNCH_CHECK();
   plan_items_fill_kernel<<<tamx::kScanBlocks, kPlanThreads, 0, s>>>(
       wl->tasks, wl->counters, bm, bn, wl->task_capacity, partial, wl->item_prefix,
-      wl->item_task, wl->item_capacity);
+      wl->item_task, wl->item_capacity, wl->queue);
   TAMX_LAUNCH_CHECK();
   return TAMX_OK;
 }

@@ -24,6 +24,7 @@
 
 #include "tamx_internal.hpp"
 #include "tamx_map.hpp"
+#include "tamx_queue.hpp"
 
 namespace {
 
@@ -94,7 +95,6 @@ template <>
 __device__ inline float buffer_load<float>(__amdgpu_buffer_rsrc_t d, uint32_t off) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(d, off, 0, 0));
 }
-constexpr int kRegions = 8;   // XCDs of an MI355X; the queue holds kRegions + 1 counters
 constexpr int kPairWin = 64;  // pair descriptors staged in LDS at a time
 
 // the address out-of-tile lanes load from
@@ -159,29 +159,9 @@ __global__ __launch_bounds__(kThreads, (sizeof(T) == 8 && BM == 64 && BN == 64 &
   const int32_t ntasks = uni((int32_t)ntasks64);
   const int32_t total = uni(p.prefix[ntasks > 0 ? ntasks : 0]);
 
-  // Items are split into kRegions contiguous ranges, one per XCD: a
-  // workgroup drains the range of its own XCD (workgroups are dispatched to
-  // XCDs round-robin by blockIdx), so the macro tiles of one result tile,
-  // which share A and B panels, run on one L2; then it steals from the
-  // other ranges in turn.
-  const int home = blockIdx.x % kRegions;
-  int tried = 0;  // used by thread 0 only
+  tamx::ItemQueue queue(p.queue, total);  // used by thread 0 only
   for (;;) {
-    if (tid == 0) {
-      int it = -1;
-      while (tried < kRegions) {
-        const int r = (home + tried) % kRegions;
-        const int rb = (int)((int64_t)total * r / kRegions);
-        const int re = (int)((int64_t)total * (r + 1) / kRegions);
-        const int q = rb < re ? atomicAdd(&p.queue[r], 1) : 0;
-        if (rb + q < re) {
-          it = rb + q;
-          break;
-        }
-        ++tried;
-      }
-      s_item = it;
-    }
+    if (tid == 0) s_item = queue.next();
     __syncthreads();
     const int item = uni(s_item);
     __syncthreads();
@@ -546,15 +526,6 @@ __global__ __launch_bounds__(kThreads, (sizeof(T) == 8 && BM == 64 && BN == 64 &
             }
           }
     });
-  }
-
-  if (tid == 0) {
-    __threadfence();
-    const int done = atomicAdd(&p.queue[kRegions], 1);
-    if (done == (int)gridDim.x - 1) {
-      // last workgroup out: every grab has happened, reset for the next launch
-      for (int r = 0; r <= kRegions; ++r) atomicExch(&p.queue[r], 0);
-    }
   }
 }
 

@@ -61,14 +61,14 @@ struct tamx_worklist {
   int64_t* tile_volume = nullptr;
   int64_t* tile_flops = nullptr;
   // scratch of the grouped GEMM: macro-tile prefix over tasks and the
-  // persistent-kernel queue (next item, finished workgroups)
+  // persistent kernel's item counters
   int32_t* item_prefix = nullptr;  // task_capacity + 1
   // position of each task's result tile in the grid (written by
   // tamx_contraction_worklist; read by launches with a scatter plan)
   int32_t* task_tile = nullptr;
   int32_t* item_task = nullptr;    // item -> task map, item_capacity entries
   int64_t item_capacity = 0;
-  int32_t* queue = nullptr;        // 16 int32 (per-XCD next item, done count), zero between launches
+  int32_t* queue = nullptr;        // item counters (tamx_queue.hpp), cleared by plan_items
   // partial sums of the multi-workgroup scans: max(kScanBlocks, grid tiles
   // / 256 + 1) + 1 entries of 32 bytes
   void* scan_partials = nullptr;
@@ -79,8 +79,9 @@ constexpr int kScanBlocks = 256;  // workgroups of the multi-workgroup scans
 
 // Fills wl->item_prefix (macro tiles of bm x bn per task, exclusive prefix,
 // total at [ntasks]) and wl->item_task (item -> task) when the total fits
-// wl->item_capacity.  Three launches on `s`; reads the task count from the
-// work list's counters, so the sequence is graph-capturable.
+// wl->item_capacity, and clears the item queue.  Three launches on `s`;
+// reads the task count from the work list's counters, so the sequence is
+// graph-capturable.
 int plan_items(tamx_worklist* wl, int bm, int bn, hipStream_t s);
 // Resolves ctx->norm_scratch on ctx's device (which must be current).
 int norm_scratch_address(tamx_context* ctx);

@@ -9,6 +9,7 @@
 
 #include "tamx_internal.hpp"
 #include "tamx_map.hpp"
+#include "tamx_queue.hpp"
 
 namespace tamx {
 namespace split {
@@ -61,7 +62,6 @@ struct SplitParams {
 };
 
 constexpr int kThreads = 256;
-constexpr int kRegions = 8;     // XCDs of an MI355X; the queue holds kRegions + 1 counters
 constexpr int SBK = 32;         // K per chunk (one BF16 MFMA 16x16x32)
 constexpr int kFoldChunks = 4;  // fold FP32 levels into FP64 every 128 k
 // INT8 limbs: K per chunk (one INT8 MFMA 16x16x64); the INT32 levels are

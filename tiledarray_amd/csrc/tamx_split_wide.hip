@@ -44,25 +44,10 @@ __global__ __launch_bounds__(kThreads, 1) void split_gemm_wide_kernel(SplitParam
     ntasks64 = 0;
   const int32_t ntasks = uni((int32_t)ntasks64);
   const int32_t total = uni(p.prefix[ntasks > 0 ? ntasks : 0]);
-  const int home = blockIdx.x % kRegions;
-  int tried = 0;
+  tamx::ItemQueue queue(p.queue, total);  // used by thread 0 only
   for (;;) {
     __syncthreads();  // every wave is done with the LDS buffers
-    if (tid == 0) {
-      int it = -1;
-      while (tried < kRegions) {
-        const int r = (home + tried) % kRegions;
-        const int rb = (int)((int64_t)total * r / kRegions);
-        const int re = (int)((int64_t)total * (r + 1) / kRegions);
-        const int q = rb < re ? atomicAdd(&p.queue[r], 1) : 0;
-        if (rb + q < re) {
-          it = rb + q;
-          break;
-        }
-        ++tried;
-      }
-      *s_item = it;
-    }
+    if (tid == 0) *s_item = queue.next();
     __syncthreads();
     const int item = uni(*s_item);
     __syncthreads();
@@ -311,14 +296,6 @@ __global__ __launch_bounds__(kThreads, 1) void split_gemm_wide_kernel(SplitParam
             }
           }
     });
-  }
-
-  if (tid == 0) {
-    __threadfence();
-    const int done = atomicAdd(&p.queue[kRegions], 1);
-    if (done == (int)gridDim.x - 1) {
-      for (int r = 0; r <= kRegions; ++r) atomicExch(&p.queue[r], 0);
-    }
   }
 }
 
