@@ -1,6 +1,6 @@
 // Plain entry points of the grouped GEMM and its item planner (the kernel
 // is in tamx_gemm.hpp).
-#include "tamx_gemm.hpp"
+#include "tamx_gemm_plain.hpp"
 #include "tamx_queue.hpp"
 #include "tamx_scan.hpp"
 

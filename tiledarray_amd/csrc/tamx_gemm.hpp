@@ -1,6 +1,7 @@
-// The persistent grouped GEMM kernel (FP64 and FP32 MFMA), shared by the
-// plain entry points (tamx_gemm.hip) and the gathered ones
-// (tamx_gemm_gather.hip).
+// The persistent grouped GEMM (FP64 and FP32 MFMA): what its two kernels
+// share, the launches, and the kernel for gathered operands
+// (tamx_gemm_gather.hip); the kernel for plain operands is in
+// tamx_gemm_plain.hpp.
 //
 // One launch computes every result tile of a contraction.  A result tile of
 // m x n is cut into BM x BN macro tiles ("items"); a workgroup takes items
@@ -78,23 +79,6 @@ struct GemmParams {
 
 constexpr int kThreads = 256;
 
-// Buffer loads of plain operands: descriptor word 3 for raw 32-bit-format
-// buffers on this family, the offset that lies outside every range, and the
-// largest leading dimension whose per-element offsets stay below it.
-constexpr int kBufFlags = 0x00020000;
-constexpr uint32_t kOutside = 0x80000000u;
-constexpr int kBufLd = 1 << 20;
-
-template <typename T>
-__device__ inline T buffer_load(__amdgpu_buffer_rsrc_t d, uint32_t off);
-template <>
-__device__ inline double buffer_load<double>(__amdgpu_buffer_rsrc_t d, uint32_t off) {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(d, off, 0, 0));
-}
-template <>
-__device__ inline float buffer_load<float>(__amdgpu_buffer_rsrc_t d, uint32_t off) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(d, off, 0, 0));
-}
 constexpr int kPairWin = 64;  // pair descriptors staged in LDS at a time
 
 // the address out-of-tile lanes load from
@@ -114,15 +98,17 @@ __device__ inline int64_t uni64(int64_t x) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// GM: which operands the launch gathers (bit 0 A, bit 1 B; 0 for the plain
-// kernel).  A gathered operand's tile t is read through p.a_gather[t] (or
-// p.b_gather[t]), element (row, k) at the pair's tile offset + rowoff(row)
+// GM: which operands the launch gathers (bit 0 A, bit 1 B).  A gathered
+// operand's tile t is read through p.a_gather[t] (or p.b_gather[t]), element (row, k) at the pair's tile offset + rowoff(row)
 // + koff(k), instead of through the pair's leading dimension.  TA / TB then
 // pick only which index the staging lanes run along (A: NoTrans k, Trans m;
 // B: NoTrans n, Trans k).
 template <typename T, int BM, int BN, int BK, bool TA, bool TB, int GM>
-__global__ __launch_bounds__(kThreads, (sizeof(T) == 8 && BM == 64 && BN == 64 && BK == 16) ? 4 : 1) void grouped_gemm_kernel(GemmParams<T> p) {
-  constexpr bool GA = (GM & 1) != 0, GB = (GM & 2) != 0, G = GM != 0;
+__global__ __launch_bounds__(kThreads,
+                             (sizeof(T) == 8 && BM == 64 && BN == 64 && BK == 16) ? 4 : 1)
+void grouped_gemm_kernel(GemmParams<T> p) {
+  constexpr bool GA = (GM & 1) != 0, GB = (GM & 2) != 0;
+  static_assert(GM != 0, "plain operands have their own kernel");
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
   constexpr int FM = BM / 32, FN = BN / 32;  // 16x16 blocks per wave (2x2 waves)
@@ -210,15 +196,6 @@ __global__ __launch_bounds__(kThreads, (sizeof(T) == 8 && BM == 64 && BN == 64 &
     int a_lda = 0, b_ldb = 0, pk = 0;
     int64_t a_off[A_LD], b_off[B_LD];
     bool a_ok[A_LD], b_ok[B_LD];
-    // Plain operands are read with buffer loads: per chunk one descriptor
-    // per operand based at the macro tile's first row (column) and the
-    // chunk's first k, and per element a 32-bit byte offset from it that is
-    // fixed for the pair.  An element outside the tile carries kOutside,
-    // beyond every descriptor's range, and loads zero; so do the k rows past
-    // the pair's end where k is the slow index (the range stops there).
-    // Pairs with a leading dimension above kBufLd take the pointer path.
-    uint32_t a_vo[A_LD], b_vo[B_LD];
-    bool buf_ok = false;
     // k-mode maps of the current pair's gathered tiles
     tamx::GatherMode ga_k[4], gb_k[4];
     int at = 0, bt = 0;
@@ -241,10 +218,8 @@ __global__ __launch_bounds__(kThreads, (sizeof(T) == 8 && BM == 64 && BN == 64 &
         pk = uni(pp.k);
         a_lda = uni(pp.lda);
         b_ldb = uni(pp.ldb);
-        if constexpr (G) {
-          at = uni(pp.a_tile);
-          bt = uni(pp.b_tile);
-        }
+        at = uni(pp.a_tile);
+        bt = uni(pp.b_tile);
       } else {
         const auto& pp = tamx::scalar_ptr(p.pairs)[pi];
         a_base = uni64(pp.a_off);
@@ -252,47 +227,29 @@ __global__ __launch_bounds__(kThreads, (sizeof(T) == 8 && BM == 64 && BN == 64 &
         pk = uni(pp.k);
         a_lda = uni(pp.lda);
         b_ldb = uni(pp.ldb);
-        if constexpr (G) {
-          at = uni(pp.a_tile);
-          bt = uni(pp.b_tile);
+        at = uni(pp.a_tile);
+        bt = uni(pp.b_tile);
+      }
+#pragma unroll
+      for (int e = 0; e < A_LD; ++e) {
+        const int slow = a_slow + e * A_STEP;
+        if (TA) {  // (k = slow, m = a_fast)
+          a_ok[e] = a_fast < mrem;
+          a_off[e] = (int64_t)slow * a_lda + r0 + a_fast;
+        } else {  // (m = slow, k = a_fast)
+          a_ok[e] = slow < mrem;
+          a_off[e] = (int64_t)(r0 + slow) * a_lda + a_fast;
         }
       }
-      if constexpr (!G) {
-        buf_ok = a_lda <= kBufLd && b_ldb <= kBufLd;
 #pragma unroll
-        for (int e = 0; e < A_LD; ++e) {
-          const int slow = a_slow + e * A_STEP;
-          const bool in = TA ? a_fast < mrem : slow < mrem;
-          a_vo[e] = in ? (uint32_t)(slow * a_lda + a_fast) * (uint32_t)sizeof(T) : kOutside;
-        }
-#pragma unroll
-        for (int e = 0; e < B_LD; ++e) {
-          const int slow = b_slow + e * B_STEP;
-          const bool in = TB ? slow < nrem : b_fast < nrem;
-          b_vo[e] = in ? (uint32_t)(slow * b_ldb + b_fast) * (uint32_t)sizeof(T) : kOutside;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < A_LD; ++e) {
-          const int slow = a_slow + e * A_STEP;
-          if (TA) {  // (k = slow, m = a_fast)
-            a_ok[e] = a_fast < mrem;
-            a_off[e] = (int64_t)slow * a_lda + r0 + a_fast;
-          } else {  // (m = slow, k = a_fast)
-            a_ok[e] = slow < mrem;
-            a_off[e] = (int64_t)(r0 + slow) * a_lda + a_fast;
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < B_LD; ++e) {
-          const int slow = b_slow + e * B_STEP;
-          if (TB) {  // (n = slow, k = b_fast)
-            b_ok[e] = slow < nrem;
-            b_off[e] = (int64_t)(c0 + slow) * b_ldb + b_fast;
-          } else {  // (k = slow, n = b_fast)
-            b_ok[e] = b_fast < nrem;
-            b_off[e] = (int64_t)slow * b_ldb + c0 + b_fast;
-          }
+      for (int e = 0; e < B_LD; ++e) {
+        const int slow = b_slow + e * B_STEP;
+        if (TB) {  // (n = slow, k = b_fast)
+          b_ok[e] = slow < nrem;
+          b_off[e] = (int64_t)(c0 + slow) * b_ldb + b_fast;
+        } else {  // (k = slow, n = b_fast)
+          b_ok[e] = b_fast < nrem;
+          b_off[e] = (int64_t)slow * b_ldb + c0 + b_fast;
         }
       }
       // gathered operands: row offsets of the thread's rows through the
@@ -341,57 +298,6 @@ __global__ __launch_bounds__(kThreads, (sizeof(T) == 8 && BM == 64 && BN == 64 &
     // pair's last chunk is zero padding, skipped)
     auto load_chunk = [&](T (&ra)[A_LD], T (&rb)[B_LD]) -> int {
       const int kc = min(BK, pk - lk0);
-      if constexpr (!G) {
-        if (buf_ok) {
-          // chunk origins (elements) and ranges (bytes): k-slow operands
-          // end at the pair's last k row, k-fast ones rely on the marks
-          const int64_t a_org = uni64(a_base + (TA ? (int64_t)lk0 * a_lda + r0
-                                                    : (int64_t)r0 * a_lda + lk0));
-          const int64_t b_org = uni64(b_base + (TB ? (int64_t)c0 * b_ldb + lk0
-                                                    : (int64_t)lk0 * b_ldb + c0));
-          const int a_rng = TA ? uni(kc * a_lda * (int)sizeof(T)) : (int)(kOutside - 1);
-          const int b_rng = TB ? (int)(kOutside - 1) : uni(kc * b_ldb * (int)sizeof(T));
-          const auto ra_d = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + a_org), (short)0,
-                                                              a_rng, kBufFlags);
-          const auto rb_d = __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + b_org), (short)0,
-                                                              b_rng, kBufFlags);
-          if (kc == BK || (TA && !TB)) {
-#pragma unroll
-            for (int e = 0; e < A_LD; ++e) ra[e] = buffer_load<T>(ra_d, a_vo[e]);
-#pragma unroll
-            for (int e = 0; e < B_LD; ++e) rb[e] = buffer_load<T>(rb_d, b_vo[e]);
-          } else {
-            // a pair's last chunk: k-fast operands mask the k past its end
-            const bool a_kok = TA || a_fast < kc, b_kok = !TB || b_fast < kc;
-#pragma unroll
-            for (int e = 0; e < A_LD; ++e) ra[e] = buffer_load<T>(ra_d, a_kok ? a_vo[e] : kOutside);
-#pragma unroll
-            for (int e = 0; e < B_LD; ++e) rb[e] = buffer_load<T>(rb_d, b_kok ? b_vo[e] : kOutside);
-          }
-        } else {
-          // 64-bit addresses, recomputed per chunk (no state kept per pair)
-          const T* __restrict__ a = p.A + a_base;
-          const T* __restrict__ b = p.B + b_base;
-#pragma unroll
-          for (int e = 0; e < A_LD; ++e) {
-            const int slow = a_slow + e * A_STEP;
-            const bool ok = TA ? (a_fast < mrem && slow < kc) : (slow < mrem && a_fast < kc);
-            const int64_t off = TA ? (int64_t)(lk0 + slow) * a_lda + r0 + a_fast
-                                   : (int64_t)(r0 + slow) * a_lda + lk0 + a_fast;
-            ra[e] = *(ok ? tamx::global_ptr(a + off) : tamx::global_ptr(zero_of<T>()));
-          }
-#pragma unroll
-          for (int e = 0; e < B_LD; ++e) {
-            const int slow = b_slow + e * B_STEP;
-            const bool ok = TB ? (slow < nrem && b_fast < kc) : (b_fast < nrem && slow < kc);
-            const int64_t off = TB ? (int64_t)(c0 + slow) * b_ldb + lk0 + b_fast
-                                   : (int64_t)(lk0 + slow) * b_ldb + c0 + b_fast;
-            rb[e] = *(ok ? tamx::global_ptr(b + off) : tamx::global_ptr(zero_of<T>()));
-          }
-        }
-        if (lp < pend) advance();
-        return uni((kc + 3) >> 2);
-      }
       const T* __restrict__ a = p.A + a_base;
       const T* __restrict__ b = p.B + b_base;
       const int64_t a_k = TA ? (int64_t)lk0 * a_lda : lk0;
@@ -533,10 +439,19 @@ struct TileCfg {
   int bm, bn;
 };
 
+// The kernel of a launch: the gathering one here; tamx_gemm_plain.hpp
+// specialises GM = 0.
+template <typename T, int BM, int BN, int BK, bool TA, bool TB, int GM>
+struct GemmKernel {
+  static constexpr auto get() { return grouped_gemm_kernel<T, BM, BN, BK, TA, TB, GM>; }
+  static constexpr int threads() { return kThreads; }
+};
+
 template <typename T, int BM, int BN, int BK, bool TA, bool TB, int GM>
 int launch_cfg(tamx_context* ctx, tamx_worklist* wl, const GemmParams<T>& prm,
                hipStream_t s, int wgs_per_cu) {
-  auto kern = grouped_gemm_kernel<T, BM, BN, BK, TA, TB, GM>;
+  using K = GemmKernel<T, BM, BN, BK, TA, TB, GM>;
+  auto kern = K::get();
   static std::mutex mu;
   static std::unordered_map<int, int> occ_cache;
   int occ = 0;
@@ -545,7 +460,7 @@ int launch_cfg(tamx_context* ctx, tamx_worklist* wl, const GemmParams<T>& prm,
     auto it = occ_cache.find(ctx->device);
     if (it == occ_cache.end()) {
       int o = 0;
-      TAMX_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kern, kThreads, 0));
+      TAMX_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kern, K::threads(), 0));
       occ_cache[ctx->device] = o > 0 ? o : 1;
       occ = occ_cache[ctx->device];
     } else {
@@ -554,7 +469,7 @@ int launch_cfg(tamx_context* ctx, tamx_worklist* wl, const GemmParams<T>& prm,
   }
   const int grid = ctx->num_cus * (wgs_per_cu > 0 ? std::min(wgs_per_cu, occ) : occ);
   if (int rc = tamx::plan_items(wl, BM, BN, s)) return rc;
-  kern<<<grid, kThreads, 0, s>>>(prm);
+  kern<<<grid, K::threads(), 0, s>>>(prm);
   TAMX_LAUNCH_CHECK();
   return TAMX_OK;
 }
