@@ -35,6 +35,7 @@ FILE_FLAGS = {"tamx_shape.hip": ["-ffp-contract=off"],
               "tamx_gemm_gather.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "tamx_gemm_gather_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "tamx_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "tamx_split_stage.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "tamx_split_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "tamx_split_i8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 

@@ -36,6 +36,8 @@ struct ItemQueue {
   int32_t total;
   int tried = 0;       // ranges found empty, starting with the own one
   bool first = true;
+  bool asked = false;  // `pending` holds an item number of the own range
+  int32_t pending = 0;
 
   __device__ ItemQueue(int32_t* counters_, int32_t total_) : counters(counters_), total(total_) {}
 
@@ -49,11 +51,15 @@ struct ItemQueue {
     }
     for (; tried < kRegions; ++tried) {
       const int r = (home + tried) % kRegions;
-      // the first item of the range that no workgroup owns
-      const int rb = range_begin(r) + (int)((gridDim.x + kRegions - 1 - r) / kRegions);
+      const int rb = owned_end(r);
       const int left = range_begin(r + 1) - rb;
       if (left <= 0) continue;
       int32_t* c = counters + r * kQueueStride;
+      if (asked) {
+        asked = false;
+        if (pending < left) return rb + pending;
+        continue;
+      }
       if (tried > 0 && __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= left)
         continue;
       const int q = atomicAdd(c, 1);
@@ -62,7 +68,24 @@ struct ItemQueue {
     return -1;
   }
 
+  // Takes the next item of the own range for next() to return.  Called
+  // shortly before an item ends, while the other waves still multiply: an item
+  // is bound to its workgroup from here on.
+  __device__ inline void prefetch() {
+    const int home = blockIdx.x % kRegions;
+    if (first || asked || tried > 0 || owned_end(home) >= range_begin(home + 1)) return;
+    pending = atomicAdd(counters + home * kQueueStride, 1);
+    // (waits here: an answer left in flight would have the compiler wait for
+    // all loads in flight wherever its register may be live)
+    asm volatile("" : "+v"(pending));
+    asked = true;
+  }
+
  private:
+  // the first item of range r that no workgroup owns
+  __device__ inline int owned_end(int r) const {
+    return range_begin(r) + (int)((gridDim.x + kRegions - 1 - r) / kRegions);
+  }
   __device__ inline int range_begin(int r) const { return (int)((int64_t)total * r / kRegions); }
 };
 

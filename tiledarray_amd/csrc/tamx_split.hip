@@ -787,11 +787,10 @@ __global__ __launch_bounds__(128 * WM, I8 ? 2 : 1) void split_gemm_kernel(SplitP
 
 template <int S, bool I8>
 int launch_split_gemm(tamx_context* ctx, tamx_worklist* wl, const SplitParams& prm,
-                      hipStream_t s, bool m32 = false, bool rows128 = false) {
-  auto kern = split_gemm_kernel<S, I8>;
+                      hipStream_t s, bool rows128 = false) {
+  auto kern = split_gemm_kernel<S, I8, I8>;  // INT8: the 32x32x32 blocks
   int threads = kThreads, bm = SBM;
   if constexpr (I8) {
-    if (m32) kern = split_gemm_kernel<S, I8, true>;
     if constexpr (S > 2)
       if (rows128) {
         kern = split_gemm_kernel<S, I8, false, 4>;
@@ -1120,7 +1119,7 @@ int tamx_split_plan_create_typed(tamx_context* ctx, int limb_type, int nslices, 
   const int transpose = is_right ? (op == 0) : (op == 1);
   std::vector<SplitTile> tiles(ntiles);
   std::vector<int64_t> prefix(ntiles + 1, 0);
-  int64_t off = 0, blocks = 0, max_kpad = 32;
+  int64_t off = 0, blocks = 0, max_kpad = 32, max_tile = 0;
   for (int64_t t = 0; t < ntiles; ++t) {
     SplitTile& st = tiles[t];
     st = SplitTile{};
@@ -1140,6 +1139,7 @@ int tamx_split_plan_create_typed(tamx_context* ctx, int limb_type, int nslices, 
     st.k_pad = std::max(kq, (st.out_k + kq - 1) / kq * kq);
     st.limb_off = off;
     off += (int64_t)nslices * st.rows_pad * st.k_pad;
+    max_tile = std::max(max_tile, off - st.limb_off);
     max_kpad = std::max<int64_t>(max_kpad, st.k_pad);
     blocks += (int64_t)((st.rows_pad + kSplitBR - 1) / kSplitBR) * split_blocks_k(st.k_pad);
   }
@@ -1151,6 +1151,7 @@ int tamx_split_plan_create_typed(tamx_context* ctx, int limb_type, int nslices, 
   plan->nslices = nslices;
   plan->limb_type = limb_type;
   plan->limb_elems = off + (int64_t)kLimbSlackRows * max_kpad * nslices;
+  plan->max_tile = max_tile;
   plan->nblocks = blocks;
   hipError_t e = hipMalloc(&plan->tiles, std::max<size_t>(1, tiles.size()) * sizeof(SplitTile));
   if (e == hipSuccess) e = hipMalloc(&plan->block_prefix, prefix.size() * sizeof(int64_t));
@@ -1205,7 +1206,7 @@ int tamx_split_plan_create_general_typed(tamx_context* ctx, int limb_type, int n
   if (int rc = tamx::activate(ctx)) return rc;
   std::vector<SplitTile> tiles(ntiles);
   std::vector<int64_t> prefix(ntiles + 1, 0);
-  int64_t off = 0, blocks = 0, max_kpad = 32;
+  int64_t off = 0, blocks = 0, max_kpad = 32, max_tile = 0;
   for (int64_t t = 0; t < ntiles; ++t) {
     SplitTile& st = tiles[t];
     st = SplitTile{};
@@ -1236,6 +1237,7 @@ int tamx_split_plan_create_general_typed(tamx_context* ctx, int limb_type, int n
     st.k_pad = std::max(kq, (st.out_k + kq - 1) / kq * kq);
     st.limb_off = off;
     off += (int64_t)nslices * st.rows_pad * st.k_pad;
+    max_tile = std::max(max_tile, off - st.limb_off);
     max_kpad = std::max<int64_t>(max_kpad, st.k_pad);
     blocks += (int64_t)((st.rows_pad + kSplitBR - 1) / kSplitBR) * split_blocks_k(st.k_pad);
   }
@@ -1247,6 +1249,7 @@ int tamx_split_plan_create_general_typed(tamx_context* ctx, int limb_type, int n
   plan->nslices = nslices;
   plan->limb_type = limb_type;
   plan->limb_elems = off + (int64_t)kLimbSlackRows * max_kpad * nslices;
+  plan->max_tile = max_tile;
   plan->nblocks = blocks;
   hipError_t e = hipMalloc(&plan->tiles, std::max<size_t>(1, tiles.size()) * sizeof(SplitTile));
   if (e == hipSuccess) e = hipMalloc(&plan->block_prefix, prefix.size() * sizeof(int64_t));
@@ -1354,6 +1357,12 @@ int tamx_grouped_gemm_split_scatter(tamx_context* ctx, tamx_worklist* wl, double
                   c_scatter ? c_scatter->tiles : nullptr,
                   wl->task_tile};
   hipStream_t s = tamx::as_stream(stream);
+  // The staged kernel addresses a tile's limbs by 32-bit offsets; tiles of
+  // 2 GB of limbs or more go to the kernels with 64-bit addresses, which give
+  // the same bits.
+  const int64_t limb_bytes = a_plan->limb_type == TAMX_LIMB_I8 ? 1 : 2;
+  const bool compact =
+      std::max(a_plan->max_tile, b_plan->max_tile) * limb_bytes < kStagedTileBytes;
   if (a_plan->limb_type == TAMX_LIMB_I8) {
     if (cfg && cfg->bm == SBM && cfg->bn == SBN && cfg->bk == 2 * SBK8)
       return launch_split_gemm_i8_2w(a_plan->nslices, ctx, wl, prm, s);
@@ -1362,24 +1371,27 @@ int tamx_grouped_gemm_split_scatter(tamx_context* ctx, tamx_worklist* wl, double
     // 128 x 64 from five limbs on: eight waves of 32 x 32 (the wide
     // kernel's 64 x 32 waves need too many accumulator registers there)
     if (cfg && cfg->bm == 2 * SBM && cfg->bn == SBN && a_plan->nslices >= 5)
-      return a_plan->nslices == 5 ? launch_split_gemm<5, true>(ctx, wl, prm, s, false, true)
-                                  : launch_split_gemm<6, true>(ctx, wl, prm, s, false, true);
+      return a_plan->nslices == 5 ? launch_split_gemm<5, true>(ctx, wl, prm, s, true)
+                                  : launch_split_gemm<6, true>(ctx, wl, prm, s, true);
     if (cfg && !(cfg->bm == SBM && cfg->bn == SBN))
       return launch_split_gemm_wide(TAMX_LIMB_I8, a_plan->nslices, cfg->bm, cfg->bn, ctx, wl,
                                     prm, s);
     // bk 64: the 32x32x32 blocks
-    const bool m32 = cfg && cfg->bk == SBK8;
+    if (!(cfg && cfg->bk == SBK8))
+      return compact ? launch_split_gemm_staged(TAMX_LIMB_I8, a_plan->nslices, ctx, wl, prm, s)
+                     : launch_split_gemm_i8_ring(a_plan->nslices, ctx, wl, prm, s);
     switch (a_plan->nslices) {
-      case 2: return launch_split_gemm<2, true>(ctx, wl, prm, s, m32);
-      case 3: return launch_split_gemm<3, true>(ctx, wl, prm, s, m32);
-      case 4: return launch_split_gemm<4, true>(ctx, wl, prm, s, m32);
-      case 5: return launch_split_gemm<5, true>(ctx, wl, prm, s, m32);
-      default: return launch_split_gemm<6, true>(ctx, wl, prm, s, m32);
+      case 2: return launch_split_gemm<2, true>(ctx, wl, prm, s);
+      case 3: return launch_split_gemm<3, true>(ctx, wl, prm, s);
+      case 4: return launch_split_gemm<4, true>(ctx, wl, prm, s);
+      case 5: return launch_split_gemm<5, true>(ctx, wl, prm, s);
+      default: return launch_split_gemm<6, true>(ctx, wl, prm, s);
     }
   }
   if (cfg && !(cfg->bm == SBM && cfg->bn == SBN))
     return launch_split_gemm_wide(TAMX_LIMB_BF16, a_plan->nslices, cfg->bm, cfg->bn, ctx, wl,
                                   prm, s);
+  if (compact) return launch_split_gemm_staged(TAMX_LIMB_BF16, a_plan->nslices, ctx, wl, prm, s);
   switch (a_plan->nslices) {
     case 2: return launch_split_gemm<2, false>(ctx, wl, prm, s);
     case 3: return launch_split_gemm<3, false>(ctx, wl, prm, s);

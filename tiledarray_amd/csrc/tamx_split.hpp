@@ -98,6 +98,14 @@ __device__ inline int64_t uni64(int64_t x) {
 // write do too).
 __device__ inline int lds_unit(int r, int q) { return r * 4 + (q ^ ((r >> 1) & 3)); }
 
+// The grouped split GEMM with 64 x 64 macro tiles for 2 to 6 BF16 or INT8
+// limbs on the 16-row MFMA, chunks multiplied out of registers
+// (tamx_split_stage.hip); plans its items and launches.  Addresses inside a
+// tile's limbs are 32-bit offsets: every tile's limbs must stay below
+// kStagedTileBytes.
+constexpr int64_t kStagedTileBytes = int64_t(1) << 31;
+int launch_split_gemm_staged(int limb_type, int nslices, tamx_context* ctx, tamx_worklist* wl,
+                             const SplitParams& prm, hipStream_t s);
 // The grouped split GEMM with a bm x bn macro tile of 128 x 64 or 64 x 128
 // for 2 to 4 limbs (tamx_split_wide.hip); plans its items and launches.
 int launch_split_gemm_wide(int limb_type, int nslices, int bm, int bn, tamx_context* ctx,
@@ -122,6 +130,7 @@ struct tamx_split_plan {
   int32_t nslices = 0;
   int32_t limb_type = 0;    // TAMX_LIMB_BF16 or TAMX_LIMB_I8
   int64_t limb_elems = 0;   // size of the limb pool in limbs (bf16 or int8)
+  int64_t max_tile = 0;     // limbs of the largest tile (all planes)
   int64_t nblocks = 0;      // 16 x 128 blocks of the limb layouts over all tiles
   tamx::split::SplitTile* tiles = nullptr;  // device
   int64_t* block_prefix = nullptr;          // device, ntiles + 1
