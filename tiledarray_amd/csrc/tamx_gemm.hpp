@@ -20,6 +20,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <unordered_map>
 
@@ -488,8 +489,37 @@ constexpr int kConfigs[][3] = {{64, 64, 16}, {64, 64, 32}, {128, 128, 16},
                                {128, 64, 16}, {64, 128, 16}, {32, 32, 16},
                                {32, 32, 32}, {128, 64, 32}, {64, 128, 32}};
 
-// One launch of the grouped GEMM with the configuration `cfg` (null: the
-// default 64 x 64 x 16).  GM: which operands are gathered (0: none).  The
+// The macro tile of a launch without a configuration.
+//  - Gathered operands: 64 x 64 x 16.
+//  - FP32: 64 x 64 x 32, whose chunks are as many bytes as FP64's of 16 k:
+//    half the barriers, and twice the bytes of a row per load (GEMM of 1024
+//    tensor-of-tensor products 1124 -> 1046 us, of 1501 x 1777 x 1300 161 ->
+//    148).
+//  - FP64: 128 x 128 x 16 reads half the operand bytes per MFMA, from LDS and
+//    from L2, but wants result tiles of many macro tiles, and enough of them
+//    that the items of a full result fill the CUs about as evenly: ladder at
+//    32 x 192, tiles of 256 x 4096 on average, a whole pass 55.4 -> 51.3 ms
+//    against 64 x 64 x 16; block-sparse 16384^3, tiles of 160, GEMM 3.39 and
+//    3.19 ms alone but no gain within a pass.  (64 x 128 x 16 gained 7 to 12%
+//    where the GEMM was repeated on operands at rest in the caches, tiles of
+//    124 and 128, and lost 3 to 7% within whole passes: 2048^3 306 -> 316 us,
+//    5000^3 730 -> 782.)
+// Every macro tile adds the same products in the same order.
+template <typename T, int GM>
+tamx_gemm_config default_config(const tamx_context* ctx, const tamx_worklist* wl) {
+  tamx_gemm_config best{64, 64, GM == 0 && sizeof(T) == 4 ? 32 : 16, 0};
+  if (GM != 0 || sizeof(T) == 4 || wl->c_tiles <= 0) return best;
+  const int64_t mean = wl->c_elems / wl->c_tiles;  // elements of a result tile
+  auto value = [&](int bm, int bn, double rate) {
+    const double per_cu = std::max(1.0, (double)wl->c_elems / (bm * bn)) / ctx->num_cus;
+    return rate * per_cu / std::ceil(per_cu);
+  };
+  if (mean >= 256 * 256 && value(128, 128, 1.1) > value(64, 64, 1.0)) best.bm = best.bn = 128;
+  return best;
+}
+
+// One launch of the grouped GEMM with the configuration `cfg` (null:
+// default_config).  GM: which operands are gathered (0: none).  The
 // gathered kernels are compiled for the three macro tiles that suit large
 // tiles (64 x 64, 128 x 64 and 64 x 128, BK 16).
 template <typename T, int GM>
@@ -507,8 +537,8 @@ int grouped_gemm(tamx_context* ctx, tamx_worklist* wl, int op_a, int op_b,
                     wl->task_capacity, wl->item_capacity, alpha, a_gather, b_gather,
                     c_scatter, wl->task_tile};
   hipStream_t s = tamx::as_stream(stream);
-  const int bm = cfg ? cfg->bm : 64, bn = cfg ? cfg->bn : 64, bk = cfg ? cfg->bk : 16;
-  const int w = cfg ? cfg->wgs_per_cu : 0;
+  const tamx_gemm_config use = cfg ? *cfg : default_config<T, GM>(ctx, wl);
+  const int bm = use.bm, bn = use.bn, bk = use.bk, w = use.wgs_per_cu;
 #define TAMX_CFG(BM_, BN_, BK_) \
   if (bm == BM_ && bn == BN_ && bk == BK_) return launch_ops<T, BM_, BN_, BK_, GM>(ctx, wl, op_a, op_b, prm, s, w);
   TAMX_CFG(64, 64, 16)

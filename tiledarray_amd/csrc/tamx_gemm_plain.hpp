@@ -385,10 +385,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void plain_gemm_kernel(GemmParam
   }
 }
 
-// workgroups per CU that the registers are budgeted for
+// workgroups per CU that the registers are budgeted for (FP32 stages of 32 k
+// are half the size of FP64's, so four of them fit)
 template <typename T>
 constexpr int plain_occupancy(int bm, int bn, int bk) {
-  if (bm * bn <= 64 * 64) return bk > 16 ? 2 : 4;
+  if (bm * bn <= 64 * 64) return bk > 16 && sizeof(T) == 8 ? 2 : 4;
   return bm * bn >= 128 * 128 ? 2 : (bk > 16 ? 1 : 3);
 }
 template <typename T, int BM, int BN, int BK, bool TA, bool TB>

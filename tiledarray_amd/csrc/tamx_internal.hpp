@@ -56,6 +56,9 @@ struct tamx_worklist {
   int64_t task_capacity = 0;
   int64_t pair_capacity = 0;
   int64_t grid_capacity = 0;
+  // elements and tiles of the result the list was last built for (0: filled
+  // by hand); only the choice of a macro tile looks at them
+  int64_t c_elems = 0, c_tiles = 0;
   // scratch of the work-list builder (per result tile of the grid)
   int32_t* tile_npairs = nullptr;
   int64_t* tile_volume = nullptr;
