@@ -65,25 +65,18 @@ constexpr int kJoinChunks = 7;
 constexpr double kJoin = 6755399441055744.0;  // 1.5 * 2^52
 constexpr int64_t kJoinBits = 0x4338000000000000;
 
-// kJoinBits + a, and x + a * b (one instruction each)
-__device__ __forceinline__ int64_t join_first(int a) {
-#ifdef __HIP_DEVICE_COMPILE__
-  int64_t r;
-  asm("v_mad_i64_i32 %0, vcc, %1, 1, %2" : "=v"(r) : "v"(a), "s"(kJoinBits) : "vcc");
-  return r;
-#else
-  return kJoinBits + a;
-#endif
-}
+// kJoinBits + a, and x + a * b, one v_mad_i64_i32 each: a factor the compiler
+// cannot see through keeps it from shifting and adding instead.  (The
+// instruction is the compiler's, not inline asm: a vector instruction has to
+// keep its distance from the MFMA whose result it reads, which the hardware
+// does not check and the compiler sees to for its own instructions only.)
 __device__ __forceinline__ int64_t join_next(int a, int b, int64_t x) {
 #ifdef __HIP_DEVICE_COMPILE__
-  int64_t r;
-  asm("v_mad_i64_i32 %0, vcc, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(x) : "vcc");
-  return r;
-#else
-  return x + (int64_t)a * b;
+  asm("" : "+s"(b));
 #endif
+  return x + (int64_t)a * b;
 }
+__device__ __forceinline__ int64_t join_first(int a) { return join_next(a, 1, kJoinBits); }
 
 // The LDS unit of a plane that holds unit q of row r.  BF16: lds_unit.  INT8:
 // the 32-k blocks of the limb layout one after the other: each group of four lanes then loads 64 consecutive
