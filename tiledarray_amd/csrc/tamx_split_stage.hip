@@ -212,7 +212,8 @@ __global__ __launch_bounds__(kThreads, staged_occupancy(S)) void split_gemm_stag
     [[maybe_unused]] int64_t a_base = 0, b_base = 0;
     uint32_t a_vo = kOutside, b_vo = kOutside;
     [[maybe_unused]] uint32_t va = kOutside, vb = kOutside;
-    [[maybe_unused]] int a_so = 0, b_so = 0, a_plane = 0, b_plane = 0;
+    // (unsigned: past a chunk's last plane they may reach 2^31)
+    [[maybe_unused]] uint32_t a_so = 0, b_so = 0, a_plane = 0, b_plane = 0;
     // per stage: whether it holds a chunk, whether that ends a pair, and the
     // pair's scale exponent
     bool valid0 = false, valid1 = false;
@@ -223,6 +224,10 @@ __global__ __launch_bounds__(kThreads, staged_occupancy(S)) void split_gemm_stag
       if constexpr (decltype(X)::value == 0) valid0 = valid; else valid1 = valid;
       if (!valid) {
         va = vb = kOutside;
+        // (the range check takes the scalar offset from the descriptor's
+        // size: left where the last chunk's loads ended, plane by plane
+        // beyond the tile, it passes 2^31 for tiles with 0.7 GB of limbs)
+        a_so = b_so = 0;
         if (tid == 0) queue.prefetch();
         return;
       }
