@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "tamx_internal.hpp"
+#include "tamx_offsets.hpp"
 #include "tamx_scan.hpp"
 #include "tamx_split.hpp"
 
@@ -84,19 +85,6 @@ __global__ void zero_u64_kernel(unsigned long long* p, int64_t n) {
   if (i < n) p[i] = 0ull;
 }
 
-// Offset of index x over n modes (extents ext, strides str, the last fastest).
-__device__ inline int64_t mixed_radix_offset(int x, int n, const int32_t* ext,
-                                             const int64_t* str) {
-  int64_t off = 0;
-  for (int d = n - 1; d > 0; --d) {
-    const int e = ext[d];
-    const int q = x / e;
-    off += (int64_t)(x - q * e) * str[d];
-    x = q;
-  }
-  return off + (int64_t)x * str[0];
-}
-
 // A block is read with the lanes along the stored rows (a transposed tile,
 // or a general one whose last row mode is the source's stride-1 mode:
 // element j of thread tid is row tid % 16, k tid / 16 + 16 j) or along k
@@ -115,9 +103,9 @@ __device__ inline bool lanes_along_rows(const SplitTile& t) {
 constexpr int kSplitOffsets = kSplitBK + kSplitBR;
 __device__ inline void offset_table(const SplitTile& t, int r0, int k0, int64_t* offs) {
   const int i = threadIdx.x;
-  if (i < kSplitBK) offs[i] = mixed_radix_offset(k0 + i, t.gen_nk, t.gk_ext, t.gk_str);
+  if (i < kSplitBK) offs[i] = mixed_radix_offset(k0 + i, t.out_k, t.gen_nk, t.gk_ext, t.gk_str);
   else if (i < kSplitOffsets)
-    offs[i] = mixed_radix_offset(r0 + i - kSplitBK, t.gen_nr, t.gr_ext, t.gr_str);
+    offs[i] = mixed_radix_offset(r0 + i - kSplitBK, t.out_rows, t.gen_nr, t.gr_ext, t.gr_str);
 }
 
 // Global loads of thread tid's 8 elements of block (r0, k0), zero outside
