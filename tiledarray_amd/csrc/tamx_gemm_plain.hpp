@@ -29,12 +29,13 @@
 
 namespace {
 
-// Buffer descriptor word 3 for raw 32-bit-format buffers on this family, the
-// offset that lies outside every range, and the largest leading dimension
-// whose per-element offsets stay below it.
+// Buffer descriptor word 3 for raw 32-bit-format buffers on this family, and
+// the offset that lies outside every range.
 constexpr int kBufFlags = 0x00020000;
 constexpr uint32_t kOutside = 0x80000000u;
-constexpr int kBufLd = 1 << 20;
+
+// what the units outside a tile load where they have 64-bit addresses
+__device__ __align__(16) const unsigned char g_zero_unit[16] = {};
 
 // Where the elements of one operand's chunk (R rows or columns of the
 // macro tile, BK k) lie in its LDS stage.  The stage is an array of 16-byte
@@ -53,6 +54,9 @@ struct StageMap {
   static constexpr int UNITS = R * BK / EPU;
   static constexpr int LOADS = (UNITS + NT - 1) / NT;
   static_assert(UNITS % 64 == 0 && UPR >= 1, "chunk split over the waves");
+  // the largest leading dimension for which a chunk's rows lie within
+  // kOutside bytes (2^22 for 64 rows of FP64)
+  static constexpr int MAX_LD = (int)(kOutside / ((KF ? R : BK) * sizeof(T)));
   static constexpr int RPW = UPR * 16 >= 256 ? 1 : 256 / (UPR * 16);  // rows per window
   __device__ static inline int swz(int r) {
     // KF: 16 rows read the same unit column; else 16 / EPU consecutive units
@@ -80,9 +84,9 @@ struct StageMap {
 };
 
 // LDS byte offsets of a wave's fragments, W waves along the direction: at(s,
-// i) is element (x0 + 16 W i, k 4 s + lk) of the stage, x0 the lane's row (column) in the wave's first
-// block.  With k contiguous the swizzle mixes s into the offset (one register
-// per step), else it mixes at most i.
+// i) is element (x0 + 16 W i, k 4 s + lk) of the stage, x0 the lane's row
+// (column) in the wave's first block.  With k contiguous the swizzle mixes s
+// into the offset (one register per step), else it mixes at most i.
 template <typename T, int R, int BK, bool KF, int NT, int W>
 struct FragMap {
   using S = StageMap<T, R, BK, KF, NT>;
@@ -118,40 +122,50 @@ __device__ __forceinline__ void load_operand(const T* base, int64_t org, int ld,
                                              const uint32_t (&vo)[S::LOADS], unsigned char* dst,
                                              int tid, int wave) {
 #ifdef __HIP_DEVICE_COMPILE__  // (the host pass does not accept the LDS load builtin)
-  if (__builtin_expect(ld <= kBufLd, 1)) {
-    const int rng =
-        kc > 0 ? uni((KF ? (rem - 1) * ld + kc : (kc - 1) * ld + rem) * (int)sizeof(T)) : 0;
-    const auto d = __builtin_amdgcn_make_buffer_rsrc((void*)(base + uni64(org)), (short)0, rng,
-                                                     kBufFlags);
-    const bool cut = KF && kc < BK;
+  const int rng =
+      kc > 0 ? uni((KF ? (rem - 1) * ld + kc : (kc - 1) * ld + rem) * (int)sizeof(T)) : 0;
+  const auto d = __builtin_amdgcn_make_buffer_rsrc((void*)(base + uni64(org)), (short)0, rng,
+                                                   kBufFlags);
+  const bool cut = KF && kc < BK;
+  asm volatile("" : "+s"(wave));  // (else every load's destination stays in a register)
 #pragma unroll
-    for (int e = 0; e < S::LOADS; ++e) {
-      if (!S::has(wave, e)) continue;
-      uint32_t o = vo[e];
-      if (cut && S::unit(tid, e) * S::EPU >= kc) o = kOutside;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          d, (__attribute__((address_space(3))) void*)(dst + (e * NT + wave * 64) * 16), 16, o, 0,
-          0, 0);
-    }
-  } else {
-    // a descriptor per stage row, based at the row
-    constexpr int RW = S::UPR < 64 ? 64 / S::UPR : 1;  // stage rows of one wave's load
-#pragma unroll 1
-    for (int e = 0; e < S::LOADS; ++e) {
-      if (!S::has(wave, e)) continue;
-      const int r_first = (e * NT + wave * 64) / S::UPR;
-#pragma unroll 1
-      for (int q = 0; q < RW; ++q) {
-        const int r = r_first + q;
-        const bool in = r < (KF ? rem : kc);
-        const int rng = in ? uni((KF ? kc : rem) * (int)sizeof(T)) : 0;
-        const auto d = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(base + uni64(org + (int64_t)r * ld)), (short)0, rng, kBufFlags);
-        if (S::row(tid, e) == r)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              d, (__attribute__((address_space(3))) void*)(dst + (e * NT + wave * 64) * 16), 16,
-              S::unit(tid, e) * 16, 0, 0, 0);
-      }
+  for (int e = 0; e < S::LOADS; ++e) {
+    if (!S::has(wave, e)) continue;
+    uint32_t o = vo[e];
+    if (cut && S::unit(tid, e) * S::EPU >= kc) o = kOutside;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        d, (__attribute__((address_space(3))) void*)(dst + (e * NT + wave * 64) * 16), 16, o, 0, 0,
+        0);
+  }
+#endif
+}
+
+// The same with 64-bit addresses, for any leading dimension.  Units outside
+// the tile load zeros; the elements of a unit that the end of its row cuts
+// are copied one by one, so that nothing past the row is read.
+template <class S, typename T, bool KF, int NT>
+__device__ __forceinline__ void load_operand_far(const T* base, int64_t org, int ld, int rem,
+                                                 int kc, unsigned char* dst, int tid, int wave) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const int rows = KF ? rem : kc, cols = KF ? kc : rem;
+#pragma unroll
+  for (int e = 0; e < S::LOADS; ++e) {
+    if (!S::has(wave, e)) continue;
+    const int r = S::row(tid, e), c = S::unit(tid, e) * S::EPU;
+    const T* src = base + org + ((int64_t)r * ld + c);
+    const bool whole = r < rows && c + S::EPU <= cols;
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) void*)(whole ? (const void*)src
+                                                              : (const void*)g_zero_unit),
+        (__attribute__((address_space(3))) void*)(dst + (e * NT + wave * 64) * 16), 16, 0, 0);
+    if (cols % S::EPU != 0 && r < rows && c < cols && !whole) {
+      T* unit = reinterpret_cast<T*>(dst + (e * NT + tid) * 16);
+      T v[S::EPU];
+#pragma unroll
+      for (int x = 0; x < S::EPU; ++x) v[x] = c + x < cols ? src[x] : T(0);
+      __builtin_amdgcn_s_waitcnt(kWaitVm0);  // (the zeros have landed)
+#pragma unroll
+      for (int x = 0; x < S::EPU; ++x) unit[x] = v[x];
     }
   }
 #endif
@@ -232,135 +246,167 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void plain_gemm_kernel(GemmParam
     const int ni = uni(min(FM, max(0, (mrem - wr + 16 * WM - 1) / (16 * WM))));
     const int nj = uni(min(FN, max(0, (nrem - wc + 16 * WN - 1) / (16 * WN))));
 
-    acc_t acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[i][j][v] = T(0);
+    // (not __syncthreads: its release fence would also wait for the loads
+    // of the next chunk; LDS stores of this thread are waited for here)
+    auto barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
+    // The item's sum, with loads through 32-bit offsets, or (FAR) 64-bit
+    // addresses where these do not do; false where a pair would need the latter.
+    //
     // Load cursor: pair lp at k lk0.  Per pair every staged unit has a
     // 32-bit byte offset from the chunk's origin, fixed for the pair; the
     // descriptor of a chunk starts at the macro tile's first row (column)
     // and the chunk's first k and ends with the last valid element, so what
     // lies past it (rows past the tile, k past the pair's end where k is the
     // slow index) loads zero.  Units wholly past the row's end carry
-    // kOutside.  With a leading dimension above kBufLd the offsets of a chunk
-    // could pass 2^31: every stage row then has its own descriptor.
-    int64_t a_base = 0, b_base = 0;
-    int a_ld = 0, b_ld = 0, pk = 0;
-    uint32_t a_vo[SA::LOADS], b_vo[SB::LOADS];
-    const int pend = t_pb + t_pc;
-    auto set_pair = [&](int pi) {
-      const auto& pp = tamx::scalar_ptr(p.pairs)[pi];
-      a_base = uni64(pp.a_off);
-      b_base = uni64(pp.b_off);
-      pk = uni(pp.k);
-      a_ld = uni(pp.lda);
-      b_ld = uni(pp.ldb);
+    // kOutside.  With a leading dimension above MAX_LD the offsets of a chunk
+    // could pass 2^31: the item is then summed anew with 64-bit addresses, in
+    // a loop of its own, for the mere presence of those loads in this one
+    // costs it up to 5%.  (Figures in FP64, NN and NT, against a descriptor
+    // for every single stage row above a leading dimension of 2^20, eight
+    // masked loads in place of each where k is contiguous: M and N 1024 over K
+    // of 2^20 + 4096 in one tile 121 and 197 ms, now 49 and 55; M and N 256
+    // over K of 2^22 + 64 483 and 786, now 229 and 248.)
+    acc_t acc[FM][FN];
+    auto sum_item = [&](auto FAR_) -> bool {
+      constexpr bool FAR = decltype(FAR_)::value;
 #pragma unroll
-      for (int e = 0; e < SA::LOADS; ++e) {
-        const int r = SA::row(tid, e), c = SA::unit(tid, e) * EPU;
-        a_vo[e] = (!TA || c < mrem) ? (uint32_t)(r * a_ld + c) * (uint32_t)sizeof(T) : kOutside;
-      }
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int e = 0; e < SB::LOADS; ++e) {
-        const int r = SB::row(tid, e), c = SB::unit(tid, e) * EPU;
-        b_vo[e] = (TB || c < nrem) ? (uint32_t)(r * b_ld + c) * (uint32_t)sizeof(T) : kOutside;
-      }
-    };
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[i][j][v] = T(0);
 
-    int lp = t_pb, lk0 = 0;
-    if (lp < pend) set_pair(lp);
-    // loads the cursor's chunk and advances the cursor; returns the number
-    // of k in the chunk
-    auto load_chunk = [&](auto X) -> int {
-      const int kc = min(BK, pk - lk0);
-      unsigned char* st = stage(X);
-      load_operand<SA, T, BK, !TA, NT>(
-          p.A, a_base + (TA ? (int64_t)lk0 * a_ld + r0 : (int64_t)r0 * a_ld + lk0), a_ld, mrem, kc,
-          a_vo, st, tid, wave);
-      load_operand<SB, T, BK, TB, NT>(
-          p.B, b_base + (TB ? (int64_t)c0 * b_ld + lk0 : (int64_t)lk0 * b_ld + c0), b_ld, nrem, kc,
-          b_vo, st + A_BYTES, tid, wave);
-      lk0 += BK;
-      if (lk0 >= pk) {
-        ++lp;
-        lk0 = 0;
-        if (lp < pend) set_pair(lp);
-      }
-      return kc;
-    };
-    // Waits for this thread's loads of a chunk of kc k, and clears what they
-    // brought from past the k end in the unit that kc cuts (the other
-    // operand holds zeros there, but zero times an infinity is not zero).
-    auto landed = [&](auto X, int kc) {
-      __builtin_amdgcn_s_waitcnt(kWaitVm0);
-      if ((!TA || TB) && (kc % EPU) != 0) {
-        unsigned char* st = stage(X);
-        auto clear = [&](auto map, unsigned char* dst) {
-          using S = decltype(map);
+      int64_t a_base = 0, b_base = 0;
+      int a_ld = 0, b_ld = 0, pk = 0;
+      uint32_t a_vo[SA::LOADS], b_vo[SB::LOADS];
+      const int pend = t_pb + t_pc;
+      int lp = t_pb, lk0 = 0;
+      bool far = false;  // a pair that needs 64-bit addresses, which ends this loop
+      auto set_pair = [&](int pi) {
+        const auto& pp = tamx::scalar_ptr(p.pairs)[pi];
+        a_base = uni64(pp.a_off);
+        b_base = uni64(pp.b_off);
+        pk = uni(pp.k);
+        a_ld = uni(pp.lda);
+        b_ld = uni(pp.ldb);
+        if (!FAR && __builtin_expect(a_ld > SA::MAX_LD || b_ld > SB::MAX_LD, 0)) {
+          far = true;
+          lp = pend;
+        }
 #pragma unroll
-          for (int e = 0; e < S::LOADS; ++e)
-            if (S::has(wave, e) && S::unit(tid, e) == kc / EPU)
-              for (int x = kc % EPU; x < EPU; ++x)
-                *reinterpret_cast<T*>(dst + (e * NT + tid) * 16 + x * (int)sizeof(T)) = T(0);
-        };
-        if constexpr (!TA) clear(SA{}, st);
-        if constexpr (TB) clear(SB{}, st + A_BYTES);
-      }
-    };
-    // (not __syncthreads: its release fence would also wait for the loads
-    // of the next chunk; LDS stores of this thread are waited for here)
-    auto barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-
-    // nks MFMA steps of a chunk; the fragments of step s + 1 are read while
-    // the MFMAs of step s run (reads of blocks past a ragged edge stay inside
-    // the stage and are not used)
-    auto compute_chunk = [&](auto X, int kc) {
-      if (ni == 0 || nj == 0) return;
-      const int nks = (kc + 3) >> 2;
-      const unsigned char* st = stage(X);
-      T af[2][FM], bf[2][FN];
-      auto frag = [&](int s, T (&a)[FM], T (&b)[FN]) {
+        for (int e = 0; e < SA::LOADS; ++e) {
+          const int r = SA::row(tid, e), c = SA::unit(tid, e) * EPU;
+          a_vo[e] = (!TA || c < mrem) ? ((uint32_t)r * a_ld + c) * (uint32_t)sizeof(T) : kOutside;
+        }
 #pragma unroll
-        for (int i = 0; i < FM; ++i) a[i] = *reinterpret_cast<const T*>(st + fa.at(s, i));
-#pragma unroll
-        for (int j = 0; j < FN; ++j) b[j] = *reinterpret_cast<const T*>(st + A_BYTES + fb.at(s, j));
+        for (int e = 0; e < SB::LOADS; ++e) {
+          const int r = SB::row(tid, e), c = SB::unit(tid, e) * EPU;
+          b_vo[e] = (TB || c < nrem) ? ((uint32_t)r * b_ld + c) * (uint32_t)sizeof(T) : kOutside;
+        }
       };
-      frag(0, af[0], bf[0]);
+
+      if (lp < pend) set_pair(lp);
+      // loads the cursor's chunk and advances the cursor; returns the number
+      // of k in the chunk
+      auto load_chunk = [&](auto X) -> int {
+        const int kc = min(BK, pk - lk0);
+        unsigned char* st = stage(X);
+        const int64_t a_org = a_base + (TA ? (int64_t)lk0 * a_ld + r0 : (int64_t)r0 * a_ld + lk0);
+        const int64_t b_org = b_base + (TB ? (int64_t)c0 * b_ld + lk0 : (int64_t)lk0 * b_ld + c0);
+        if (FAR && a_ld > SA::MAX_LD)
+          load_operand_far<SA, T, !TA, NT>(p.A, a_org, a_ld, mrem, kc, st, tid, wave);
+        else
+          load_operand<SA, T, BK, !TA, NT>(p.A, a_org, a_ld, mrem, kc, a_vo, st, tid, wave);
+        if (FAR && b_ld > SB::MAX_LD)
+          load_operand_far<SB, T, TB, NT>(p.B, b_org, b_ld, nrem, kc, st + A_BYTES, tid, wave);
+        else
+          load_operand<SB, T, BK, TB, NT>(p.B, b_org, b_ld, nrem, kc, b_vo, st + A_BYTES, tid,
+                                          wave);
+        lk0 += BK;
+        if (lk0 >= pk) {
+          ++lp;
+          lk0 = 0;
+          if (lp < pend) set_pair(lp);
+        }
+        return kc;
+      };
+      // Waits for this thread's loads of a chunk of kc k, and clears what they
+      // brought from past the k end in the unit that kc cuts (the other
+      // operand holds zeros there, but zero times an infinity is not zero).
+      auto landed = [&](auto X, int kc) {
+        __builtin_amdgcn_s_waitcnt(kWaitVm0);
+        if ((!TA || TB) && (kc % EPU) != 0) {
+          unsigned char* st = stage(X);
+          auto clear = [&](auto map, unsigned char* dst) {
+            using S = decltype(map);
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        if (s < nks) {
-          if (s + 1 < NS) frag(s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
+            for (int e = 0; e < S::LOADS; ++e)
+              if (S::has(wave, e) && S::unit(tid, e) == kc / EPU)
+                for (int x = kc % EPU; x < EPU; ++x)
+                  *reinterpret_cast<T*>(dst + (e * NT + tid) * 16 + x * (int)sizeof(T)) = T(0);
+          };
+          if constexpr (!TA) clear(SA{}, st);
+          if constexpr (TB) clear(SB{}, st + A_BYTES);
+        }
+      };
+      // nks MFMA steps of a chunk; the fragments of step s + 1 are read while
+      // the MFMAs of step s run (reads of blocks past a ragged edge stay inside
+      // the stage and are not used)
+      auto compute_chunk = [&](auto X, int kc) {
+        if (ni == 0 || nj == 0) return;
+        const int nks = (kc + 3) >> 2;
+        const unsigned char* st = stage(X);
+        T af[2][FM], bf[2][FN];
+        auto frag = [&](int s, T (&a)[FM], T (&b)[FN]) {
 #pragma unroll
-          for (int i = 0; i < FM; ++i)
+          for (int i = 0; i < FM; ++i) a[i] = *reinterpret_cast<const T*>(st + fa.at(s, i));
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-              if (i < ni && j < nj) acc[i][j] = M::op(af[s & 1][i], bf[s & 1][j], acc[i][j]);
+          for (int j = 0; j < FN; ++j)
+            b[j] = *reinterpret_cast<const T*>(st + A_BYTES + fb.at(s, j));
+        };
+        frag(0, af[0], bf[0]);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          if (s < nks) {
+            if (s + 1 < NS) frag(s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+              for (int j = 0; j < FN; ++j)
+                // (the rare loop has no conditions, for they would be held in
+                // scalar registers through the other)
+                if (FAR || (i < ni && j < nj))
+                  acc[i][j] = M::op(af[s & 1][i], bf[s & 1][j], acc[i][j]);
+          }
+        }
+      };
+
+      // Pipeline: while chunk c is multiplied out of one stage, chunk c + 1
+      // lands in the other.
+      if (lp < pend) {
+        int k0c = load_chunk(zero{}), k1c = 0;
+        for (;;) {
+          landed(zero{}, k0c);
+          barrier();
+          bool more = lp < pend;
+          if (more) k1c = load_chunk(one{});
+          compute_chunk(zero{}, k0c);
+          if (!more) break;
+          landed(one{}, k1c);
+          barrier();
+          more = lp < pend;
+          if (more) k0c = load_chunk(zero{});
+          compute_chunk(one{}, k1c);
+          if (!more) break;
         }
       }
-    };
+      return !far;
+    };  // sum_item
 
-    // Pipeline: while chunk c is multiplied out of one stage, chunk c + 1
-    // lands in the other.
-    if (lp < pend) {
-      int k0c = load_chunk(zero{}), k1c = 0;
-      for (;;) {
-        landed(zero{}, k0c);
-        barrier();
-        bool more = lp < pend;
-        if (more) k1c = load_chunk(one{});
-        compute_chunk(zero{}, k0c);
-        if (!more) break;
-        landed(one{}, k1c);
-        barrier();
-        more = lp < pend;
-        if (more) k0c = load_chunk(zero{});
-        compute_chunk(one{}, k1c);
-        if (!more) break;
-      }
+    if (__builtin_expect(!sum_item(std::false_type{}), 0)) {
+      barrier();  // every wave is done with the stages
+      (void)sum_item(std::true_type{});
     }
 
     const bool beta1 = (t_flags & TAMX_TASK_BETA1) != 0;
