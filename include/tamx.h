@@ -339,6 +339,10 @@ typedef struct tamx_gemm_config {
 } tamx_gemm_config;
 int tamx_gemm_config_count(void);
 int tamx_gemm_config_get(int index, tamx_gemm_config* cfg);
+/* The configuration that the last FP64 or FP32 grouped GEMM call on this work
+ * list ran.  Without one given, FP64 runs the macro tile that suits the list's
+ * tasks, which the device finds out; then this waits for the device. */
+int tamx_gemm_macro_tile(const tamx_worklist* wl, tamx_gemm_config* cfg);
 int tamx_grouped_gemm_f64_config(tamx_context* ctx, tamx_worklist* wl,
                                  int op_a, int op_b, double alpha,
                                  const double* A, const double* B, double* C,

@@ -126,6 +126,7 @@ SIGNATURES = {
     "tamx_grouped_gemm_f64": [_vp, _vp, _i, _i, _d, _vp, _vp, _vp, _vp],
     "tamx_gemm_config_count": [],
     "tamx_gemm_config_get": [_i, _vp],
+    "tamx_gemm_macro_tile": [_vp, _vp],
     "tamx_grouped_gemm_f64_config": [_vp, _vp, _i, _i, _d, _vp, _vp, _vp, _vp, _vp],
     "tamx_grouped_gemm_f32_config": [_vp, _vp, _i, _i, _f, _vp, _vp, _vp, _vp, _vp],
     "tamx_grouped_gemm_f32": [_vp, _vp, _i, _i, _f, _vp, _vp, _vp, _vp],

@@ -123,7 +123,8 @@ int tamx_worklist_create(tamx_context* ctx, int64_t task_capacity,
   // search over item_prefix inside the GEMM kernel
   wl->item_capacity = std::min<int64_t>(tc * 16, (int64_t(1) << 31) - 1);
   alloc(&wl->item_task, sizeof(int32_t) * wl->item_capacity);
-  alloc(&wl->queue, sizeof(int32_t) * tamx::kQueueInts);
+  alloc(&wl->queue, sizeof(int32_t) * (tamx::kQueueInts + 1));
+  wl->choice = wl->queue + tamx::kQueueInts;
   // one partial per work-list workgroup (32 result tiles each), at least
   // one per item-planner chunk
   const int64_t nparts = std::max<int64_t>(tamx::kScanBlocks, gc / 32 + 1) + 1;

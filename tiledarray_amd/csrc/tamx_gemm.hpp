@@ -20,7 +20,6 @@
 #pragma once
 
 #include <algorithm>
-#include <cmath>
 #include <mutex>
 #include <unordered_map>
 
@@ -76,6 +75,9 @@ struct GemmParams {
   // task's ldc); task_tile[t] is task t's position in the result grid
   const tamx::GatherTile* __restrict__ c_scatter;
   const int32_t* __restrict__ task_tile;
+  // the width of the macro tile that runs, where the planner picked it among
+  // those launched (null: this one)
+  const int32_t* __restrict__ choice;
 };
 
 constexpr int kThreads = 256;
@@ -100,8 +102,9 @@ __device__ inline int64_t uni64(int64_t x) {
 }
 
 // GM: which operands the launch gathers (bit 0 A, bit 1 B).  A gathered
-// operand's tile t is read through p.a_gather[t] (or p.b_gather[t]), element (row, k) at the pair's tile offset + rowoff(row)
-// + koff(k), instead of through the pair's leading dimension.  TA / TB then
+// operand's tile t is read through p.a_gather[t] (or p.b_gather[t]), element
+// (row, k) at the pair's tile offset + rowoff(row) + koff(k), instead of
+// through the pair's leading dimension.  TA / TB then
 // pick only which index the staging lanes run along (A: NoTrans k, Trans m;
 // B: NoTrans n, Trans k).
 template <typename T, int BM, int BN, int BK, bool TA, bool TB, int GM>
@@ -436,10 +439,6 @@ void grouped_gemm_kernel(GemmParams<T> p) {
   }
 }
 
-struct TileCfg {
-  int bm, bn;
-};
-
 // The kernel of a launch: the gathering one here; tamx_gemm_plain.hpp
 // specialises GM = 0.
 template <typename T, int BM, int BN, int BK, bool TA, bool TB, int GM>
@@ -451,6 +450,7 @@ struct GemmKernel {
 template <typename T, int BM, int BN, int BK, bool TA, bool TB, int GM>
 int launch_cfg(tamx_context* ctx, tamx_worklist* wl, const GemmParams<T>& prm,
                hipStream_t s, int wgs_per_cu) {
+  // (prm.choice: the items are planned already)
   using K = GemmKernel<T, BM, BN, BK, TA, TB, GM>;
   auto kern = K::get();
   static std::mutex mu;
@@ -469,7 +469,8 @@ int launch_cfg(tamx_context* ctx, tamx_worklist* wl, const GemmParams<T>& prm,
     }
   }
   const int grid = ctx->num_cus * (wgs_per_cu > 0 ? std::min(wgs_per_cu, occ) : occ);
-  if (int rc = tamx::plan_items(wl, BM, BN, s)) return rc;
+  if (prm.choice == nullptr)
+    if (int rc = tamx::plan_items(wl, BM, BN, s)) return rc;
   kern<<<grid, K::threads(), 0, s>>>(prm);
   TAMX_LAUNCH_CHECK();
   return TAMX_OK;
@@ -495,31 +496,28 @@ constexpr int kConfigs[][3] = {{64, 64, 16}, {64, 64, 32}, {128, 128, 16},
 //    half the barriers, and twice the bytes of a row per load (GEMM of 1024
 //    tensor-of-tensor products 1124 -> 1046 us, of 1501 x 1777 x 1300 161 ->
 //    148).
-//  - FP64: 128 x 128 x 16 reads half the operand bytes per MFMA, from LDS and
-//    from L2, but wants result tiles of many macro tiles, and enough of them
-//    that the items of a full result fill the CUs about as evenly: ladder at
-//    32 x 192, tiles of 256 x 4096 on average, a whole pass 55.4 -> 51.3 ms
-//    against 64 x 64 x 16; block-sparse 16384^3, tiles of 160, GEMM 3.39 and
-//    3.19 ms alone but no gain within a pass.  (64 x 128 x 16 gained 7 to 12%
-//    where the GEMM was repeated on operands at rest in the caches, tiles of
-//    124 and 128, and lost 3 to 7% within whole passes: 2048^3 306 -> 316 us,
-//    5000^3 730 -> 782.)
+//  - FP64: 64 x 64 x 16, or 128 x 128 x 16 where the planner finds that the
+//    result tiles that are there suit it (plan_choose_kernel).  Both kernels
+//    are launched and one finds no items (5 us), so this is left out where
+//    the result buffer holds less than the 3.5 macro tiles of 128 x 128 a CU
+//    that the planner asks for.  GEMM, 64 x 64 and 128 x 128: ladder at 32 x
+//    128 8.29 and 7.65 ms, dense 6144^3 in tiles of 512 7.09 and 6.82, of 320
+//    6.91 and 8.14, result tiles of 36 x 4096 0.81 and 1.02 ms.  (64 x 128 x
+//    16 gained 7 to 12% where the GEMM was repeated on operands at rest in
+//    the caches, tiles of 124 and 128, and lost 3 to 7% within whole passes:
+//    2048^3 306 -> 316 us, 5000^3 730 -> 782.)
 // Every macro tile adds the same products in the same order.
 template <typename T, int GM>
-tamx_gemm_config default_config(const tamx_context* ctx, const tamx_worklist* wl) {
-  tamx_gemm_config best{64, 64, GM == 0 && sizeof(T) == 4 ? 32 : 16, 0};
-  if (GM != 0 || sizeof(T) == 4 || wl->c_tiles <= 0) return best;
-  const int64_t mean = wl->c_elems / wl->c_tiles;  // elements of a result tile
-  auto value = [&](int bm, int bn, double rate) {
-    const double per_cu = std::max(1.0, (double)wl->c_elems / (bm * bn)) / ctx->num_cus;
-    return rate * per_cu / std::ceil(per_cu);
-  };
-  if (mean >= 256 * 256 && value(128, 128, 1.1) > value(64, 64, 1.0)) best.bm = best.bn = 128;
-  return best;
+constexpr tamx_gemm_config default_config() {
+  return {64, 64, GM == 0 && sizeof(T) == 4 ? 32 : 16, 0};
+}
+template <typename T, int GM>
+bool planner_chooses(const tamx_context* ctx, const tamx_worklist* wl) {
+  return GM == 0 && sizeof(T) == 8 && wl->c_elems >= int64_t(128 * 128 * 7 / 2) * ctx->num_cus;
 }
 
-// One launch of the grouped GEMM with the configuration `cfg` (null:
-// default_config).  GM: which operands are gathered (0: none).  The
+// One launch of the grouped GEMM with the configuration `cfg` (null: as
+// above).  GM: which operands are gathered (0: none).  The
 // gathered kernels are compiled for the three macro tiles that suit large
 // tiles (64 x 64, 128 x 64 and 64 x 128, BK 16).
 template <typename T, int GM>
@@ -535,9 +533,18 @@ int grouped_gemm(tamx_context* ctx, tamx_worklist* wl, int op_a, int op_b,
   GemmParams<T> prm{A, B, C, wl->tasks, wl->pairs, wl->counters,
                     wl->item_prefix, wl->item_task, wl->queue,
                     wl->task_capacity, wl->item_capacity, alpha, a_gather, b_gather,
-                    c_scatter, wl->task_tile};
+                    c_scatter, wl->task_tile, nullptr};
   hipStream_t s = tamx::as_stream(stream);
-  const tamx_gemm_config use = cfg ? *cfg : default_config<T, GM>(ctx, wl);
+  const tamx_gemm_config use = cfg ? *cfg : default_config<T, GM>();
+  wl->last = use;
+  wl->last_chosen = cfg == nullptr && planner_chooses<T, GM>(ctx, wl);
+  if constexpr (GM == 0 && sizeof(T) == 8)
+    if (wl->last_chosen) {
+      if (int rc = tamx::plan_items_choosing(ctx, wl, s)) return rc;
+      prm.choice = wl->choice;
+      if (int rc = launch_ops<T, 64, 64, 16, GM>(ctx, wl, op_a, op_b, prm, s, 0)) return rc;
+      return launch_ops<T, 128, 128, 16, GM>(ctx, wl, op_a, op_b, prm, s, 0);
+    }
   const int bm = use.bm, bn = use.bn, bk = use.bk, w = use.wgs_per_cu;
 #define TAMX_CFG(BM_, BN_, BK_) \
   if (bm == BM_ && bn == BN_ && bk == BK_) return launch_ops<T, BM_, BN_, BK_, GM>(ctx, wl, op_a, op_b, prm, s, w);

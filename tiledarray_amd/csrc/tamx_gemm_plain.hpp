@@ -208,7 +208,8 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void plain_gemm_kernel(GemmParam
   if (ntasks64 < 0 || ntasks64 > p.task_capacity || p.counters[TAMX_WL_STATUS] != 0)
     ntasks64 = 0;
   const int32_t ntasks = uni((int32_t)ntasks64);
-  const int32_t total = uni(p.prefix[ntasks > 0 ? ntasks : 0]);
+  int32_t total = uni(p.prefix[ntasks > 0 ? ntasks : 0]);
+  if (p.choice != nullptr && uni(*p.choice) != BM) total = 0;  // the other macro tile runs
 
   tamx::ItemQueue queue(p.queue, total);  // used by thread 0 only
   for (;;) {

@@ -56,9 +56,14 @@ struct tamx_worklist {
   int64_t task_capacity = 0;
   int64_t pair_capacity = 0;
   int64_t grid_capacity = 0;
-  // elements and tiles of the result the list was last built for (0: filled
-  // by hand); only the choice of a macro tile looks at them
-  int64_t c_elems = 0, c_tiles = 0;
+  // elements of the result buffer the list was last built for (0: filled by
+  // hand): a result that cannot be large is not offered the large macro tile
+  int64_t c_elems = 0;
+  // the last FP64 or FP32 GEMM's macro tile, and whether the planner picked
+  // its width (then in choice[0], on the device)
+  tamx_gemm_config last{};
+  bool last_chosen = false;
+  int32_t* choice = nullptr;  // behind the item counters
   // scratch of the work-list builder (per result tile of the grid)
   int32_t* tile_npairs = nullptr;
   int64_t* tile_volume = nullptr;
@@ -86,6 +91,9 @@ constexpr int kScanBlocks = 256;  // workgroups of the multi-workgroup scans
 // reads the task count from the work list's counters, so the sequence is
 // graph-capturable.
 int plan_items(tamx_worklist* wl, int bm, int bn, hipStream_t s);
+// The same for macro tiles of 64 x 64 or 128 x 128, whichever suits the list's
+// tasks better: the width goes to wl->choice on the device.
+int plan_items_choosing(tamx_context* ctx, tamx_worklist* wl, hipStream_t s);
 // Resolves ctx->norm_scratch on ctx's device (which must be current).
 int norm_scratch_address(tamx_context* ctx);
 }

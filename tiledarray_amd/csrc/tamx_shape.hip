@@ -937,7 +937,6 @@ int tamx_contraction_worklist(tamx_context* ctx,
   }
   if (int rc = tamx::activate(ctx)) return rc;
   wl->c_elems = desc->c_capacity;
-  wl->c_tiles = desc->Mt * desc->Nt * desc->nbatch;
   WlParams p{d,
              wl->tasks,
              wl->task_tile,

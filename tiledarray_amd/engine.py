@@ -721,6 +721,13 @@ class Contraction:
             t = self.tile + (16, 0)[len(self.tile) - 2:] if len(self.tile) < 4 else self.tile
             self.tile_cfg = _lib.GemmConfig(*t[:4])
 
+    def macro_tile(self):
+        """(bm, bn, bk) of the last FP64 or FP32 gemm_step; waits for the
+        device."""
+        cfg = _lib.GemmConfig()
+        call("tamx_gemm_macro_tile", self.wl.ptr, ctypes.byref(cfg))
+        return cfg.bm, cfg.bn, cfg.bk
+
     def tune(self, reps=3, force=False, warmup=True):
         """Autotunes the tile configuration on the current work list (built
         by worklist_step, with the limbs split for a split precision) and
