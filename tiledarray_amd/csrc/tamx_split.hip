@@ -361,22 +361,25 @@ void launch_split(int grid, hipStream_t s, const double* pool, const tamx_split_
 
 // ------------------------------------------------------------ the GEMM --
 
-// I8: INT8 limbs (7 bits each) on the INT8 MFMA 16x16x64 with one exact
-// INT32 accumulator per level s + t; otherwise BF16 limbs as above.  Both
-// stage 16-byte units (8 BF16 or 16 INT8 limbs of one row), 4 units of a
-// row per chunk, so the staging and the LDS layout are shared.
-// M32 (INT8 only): each wave's 32 x 32 quadrant is one block of the INT8
-// MFMA 32x32x32 instead of four of the 16x16x64 (the same products and
-// levels; on this part the 32x32x32 does twice the work in about the same
-// issue time).
+// Two LDS buffers, one or two chunks ahead, 64-bit limb addresses: BF16 limbs
+// in tiles too large for the staged kernel (tamx_split_stage.hip), INT8 limbs
+// with bk 64 (M32) and in 128 x 64 macro tiles (WM = 4).
+//
+// I8: INT8 limbs (7 bits each) on the INT8 MFMA with one exact INT32
+// accumulator per level s + t; otherwise BF16 limbs as above.  Both stage
+// 16-byte units (8 BF16 or 16 INT8 limbs of one row), 4 units of a row per
+// chunk, so the staging and the LDS layout are shared.
+// M32: each wave's 32 x 32 quadrant is one block of the INT8 MFMA 32x32x32
+// instead of four of the 16x16x64 (the same products and levels; on this part
+// the 32x32x32 does twice the work in about the same issue time).
 // WM: waves along the rows of the macro tile, 2 (64 x 64, four waves) or 4
 // (128 x 64, eight waves in one workgroup per CU: every B limb staged into
-// LDS feeds twice the rows, a quarter fewer limb bytes per product; INT8
-// limbs from three on, whose chunks are loaded straight into LDS).
+// LDS feeds twice the rows, a quarter fewer limb bytes per product; five or
+// six INT8 limbs on 16x16x64, whose chunks are loaded straight into LDS).
 template <int S, bool I8, bool M32 = false, int WM = 2>
 __global__ __launch_bounds__(128 * WM, I8 ? 2 : 1) void split_gemm_kernel(SplitParams p) {
-  static_assert(!M32 || I8, "the 32x32x32 blocks are INT8 only");
-  static_assert(WM == 2 || (WM == 4 && I8 && !M32 && S > 2), "eight waves: INT8 16x16 blocks, 3+ limbs");
+  static_assert(WM == 4 ? I8 && !M32 && S > 4 : WM == 2 && M32 == I8,
+                "eight waves: 16x16 blocks of five or six INT8 limbs");
   constexpr int BM = 32 * WM;  // macro tile rows
   constexpr int NG = I8 ? S : (S >= 3 ? 3 : S);  // BF16: P_0, P_1, P_T; INT8: levels
   constexpr int CK = I8 ? SBK8 : SBK;            // k per chunk
@@ -687,16 +690,12 @@ __global__ __launch_bounds__(128 * WM, I8 ? 2 : 1) void split_gemm_kernel(SplitP
 
     // Pipeline: registers R0/R1 hold chunks c+1 and c+2 in flight while
     // chunk c is multiplied out of LDS buffer c % 2.  One barrier per chunk.
-    // Above four limbs the second register set would cost occupancy, so the
-    // loads run one chunk ahead instead.
+    // Above four limbs the second register set would cost occupancy: the
+    // loads run one chunk ahead, straight into LDS (measured: two chunks ahead
+    // through registers is faster where it fits, 49.7 against 47.7 TFLOP/s
+    // for four BF16 limbs).
     bf8_t ra0[S], rb0[S], ra1[S], rb1[S];
-    // Above four BF16 limbs, and from three INT8 limbs on, a second
-    // register set would cost occupancy: the loads run one chunk ahead,
-    // straight into LDS (measured: two chunks ahead through registers is
-    // faster where it fits, 49.7 against 47.7 TFLOP/s for four BF16 limbs).
-    // (The 32x32x32 blocks need fewer accumulator registers: up to four
-    // INT8 limbs they keep two register sets at two waves per SIMD.)
-    constexpr bool ONE_AHEAD = I8 ? (M32 ? S > 4 : S > 2) : S > 4;
+    constexpr bool ONE_AHEAD = S > 4;
     if constexpr (ONE_AHEAD) {
       if (lp < pend) {
         load_chunk_lds(zero{});
@@ -789,14 +788,12 @@ int launch_split_gemm(tamx_context* ctx, tamx_worklist* wl, const SplitParams& p
                       hipStream_t s, bool rows128 = false) {
   auto kern = split_gemm_kernel<S, I8, I8>;  // INT8: the 32x32x32 blocks
   int threads = kThreads, bm = SBM;
-  if constexpr (I8) {
-    if constexpr (S > 2)
-      if (rows128) {
-        kern = split_gemm_kernel<S, I8, false, 4>;
-        threads = 2 * kThreads;
-        bm = 2 * SBM;
-      }
-  }
+  if constexpr (I8 && S > 4)
+    if (rows128) {
+      kern = split_gemm_kernel<S, I8, false, 4>;
+      threads = 2 * kThreads;
+      bm = 2 * SBM;
+    }
   int occ = 0;
   TAMX_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, threads, 0));
   if (occ < 1) occ = 1;
