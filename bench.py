@@ -35,9 +35,11 @@ PEAK_FP32_TFLOPS = 157.3
 # with the profile summary the counters come from; a line whose
 # configuration has no entry reports traffic null.
 TRAFFIC_BYTES = {
-    ("blocksparse", "f64", (64, 64, 16)): (4668000 * 2048 + 1006000 * 1024,
+    ("blocksparse", "f64", (64, 64, 16)): (5337000 * 2048 + 991400 * 1024,
                                            "profiles/grouped_gemm_f64_blocksparse16384.md"),
-    ("blocksparse", "i8x5", (64, 64, 16)): (2202000 * 2048 + 905900 * 1024,
+    ("blocksparse", "f64", (64, 128, 16)): (5320000 * 2048 + 996400 * 1024,
+                                            "profiles/grouped_gemm_f64_blocksparse16384.md"),
+    ("blocksparse", "i8x5", (64, 64, 16)): (1888000 * 2048 + 917000 * 1024,
                                             "profiles/split_gemm_i8x5_blocksparse16384.md"),
 }
 
@@ -114,9 +116,9 @@ def parse():
     p = argparse.ArgumentParser()
     p.add_argument("--gpus", type=int, default=1)
     p.add_argument("--steps", type=int, default=20)
-    # the GEMMs settle over their first ten or so launches (3.9 -> 3.25 ms
-    # for the block-sparse FP64 GEMM in a per-launch trace), so the default
-    # warm-up covers them
+    # the GEMMs settle over their first ten or so launches (the block-sparse
+    # FP64 GEMM by 0.6 ms in a per-launch trace), so the default warm-up
+    # covers them
     p.add_argument("--warmup", type=int, default=10)
     p.add_argument("--workload", default="blocksparse",
                    choices=["blocksparse", "dense", "ladder", "tot"])
@@ -318,7 +320,7 @@ def main():
     achieved = flops / (gemm_ms * 1e-3) / 1e12
     peak = (PEAK_FP64_TFLOPS if args.precision == "f64"
             else PEAK_INT8_TOPS if args.precision.startswith("i8") else PEAK_BF16_TFLOPS)
-    tr_bytes, tr_src = traffic(args.workload, args.precision, used_tile or [64, 64, 16])
+    tr_bytes, tr_src = traffic(args.workload, args.precision, used_tile)
 
     out = {
         "metric": METRIC,
@@ -347,7 +349,7 @@ def main():
         },
         "roofline": ({
             "bound": "mfma",
-            "kernel": f"grouped_gemm_kernel<double,{','.join(map(str, used_tile or [64, 64, 16]))}>",
+            "kernel": f"plain_gemm_kernel<double,{','.join(map(str, used_tile))}>",
             "achieved": round(achieved, 3),
             "peak": peak,
             "unit": "TFLOP/s",
