@@ -20,8 +20,8 @@
 // 16 bytes per cycle and CU, about 10 TB/s).  Staging through registers took
 // four times as many load instructions (8 bytes each) and as many LDS stores;
 // with direct loads and offsets that are fixed per pair a chunk costs no
-// vector arithmetic but the fragment addresses.  Measured against it on one
-// card: FP64 ladder at 32 x 192 53.4 -> 48.3 ms (57.6 TFLOP/s), block-sparse
+// vector arithmetic but the fragment addresses.  GEMM against it, 64 x 64 macro
+// tiles on one card: FP64 ladder at 32 x 192 53.4 -> 48.3 ms, block-sparse
 // 16384^3 3.41 -> 3.13 ms, 5000^3 700 -> 631 us.
 #pragma once
 
