@@ -101,6 +101,12 @@ def test_choice_by_what_the_screening_leaves(ctx):
         assert torch.equal(c.C[:n], C0) and bool(C0.ne(0).any())
 
 
-def test_no_launch_yet(ctx):
+def test_no_launch_yet_and_a_refused_one(ctx):
+    c = product(ctx, [64], [64])
     with pytest.raises(E._lib.TamxError):
-        product(ctx, [64], [64]).macro_tile()
+        c.macro_tile()
+    c.run()
+    c.set_tile((48, 64, 16))
+    with pytest.raises(E._lib.TamxError):
+        c.gemm_step()
+    assert c.macro_tile() == F64

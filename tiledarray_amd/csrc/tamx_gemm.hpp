@@ -473,6 +473,8 @@ int launch_cfg(tamx_context* ctx, tamx_worklist* wl, const GemmParams<T>& prm,
     if (int rc = tamx::plan_items(wl, BM, BN, s)) return rc;
   kern<<<grid, K::threads(), 0, s>>>(prm);
   TAMX_LAUNCH_CHECK();
+  wl->last = {BM, BN, BK, wgs_per_cu};
+  wl->last_chosen = prm.choice != nullptr;
   return TAMX_OK;
 }
 
@@ -536,10 +538,8 @@ int grouped_gemm(tamx_context* ctx, tamx_worklist* wl, int op_a, int op_b,
                     c_scatter, wl->task_tile, nullptr};
   hipStream_t s = tamx::as_stream(stream);
   const tamx_gemm_config use = cfg ? *cfg : default_config<T, GM>();
-  wl->last = use;
-  wl->last_chosen = cfg == nullptr && planner_chooses<T, GM>(ctx, wl);
   if constexpr (GM == 0 && sizeof(T) == 8)
-    if (wl->last_chosen) {
+    if (cfg == nullptr && planner_chooses<T, GM>(ctx, wl)) {
       if (int rc = tamx::plan_items_choosing(ctx, wl, s)) return rc;
       prm.choice = wl->choice;
       if (int rc = launch_ops<T, 64, 64, 16, GM>(ctx, wl, op_a, op_b, prm, s, 0)) return rc;
